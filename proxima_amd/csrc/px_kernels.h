@@ -168,8 +168,9 @@ hipError_t launch_flat_screen(const ScreenArgs& a, hipStream_t s);
 constexpr int kAbsMaxParts = 512;
 hipError_t launch_abs_max(const float* x, int64_t count, float* parts, int* parts_n, int* words,
                           hipStream_t s);
-// Rows [rows][dp] to fp16 copies [rows][ds] of x 2^e; max2[0], max2[1] raised to the largest
-// squared norm and squared rounding residual (float bits, in the rows' own scale).
+// Rows [rows][dp] to fp16 copies [rows][ds] of x 2^e; max2[0] raised to the largest squared norm
+// (float bits, in the rows' own scale), max2[1] to the largest squared rounding residual (in
+// that of the copy).
 hipError_t launch_screen_rows(const float* x, int64_t rows, int dp, int ds, int e,
                               unsigned short* out, int* max2, hipStream_t s);
 // The same of the rows that PQ codes [rows][m] stand for (centroids of books

@@ -555,10 +555,11 @@ __global__ __launch_bounds__(256) void abs_max_kernel(const float4* x, int64_t c
 }
 
 // One wave a row: its fp16 copy (zero pad columns), and the largest squared norm and squared
-// residual of all rows (fmax2: float bits, which order as ints where nothing is negative).
+// residual of all rows (max2: float bits, which order as ints where nothing is negative). The
+// residual is taken of the scaled row, whose values lie where squares are fp32 numbers.
 __global__ __launch_bounds__(256) void screen_rows_kernel(const float* x, int64_t rows, int dp,
-                                                          int ds, float s, float inv_s,
-                                                          unsigned short* out, int* max2) {
+                                                          int ds, float s, unsigned short* out,
+                                                          int* max2) {
     __shared__ float wn[4], wr[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float n_max = 0.f, r_max = 0.f;
@@ -569,7 +570,7 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(const float* x, int64_
         for (int c = lane * 2; c < ds; c += 128) {
             const float2 v = c < dp ? *reinterpret_cast<const float2*>(xr + c) : float2{0.f, 0.f};
             const _Float16 h0 = to_screen(v.x, s), h1 = to_screen(v.y, s);
-            const float d0 = v.x - (float)h0 * inv_s, d1 = v.y - (float)h1 * inv_s;
+            const float d0 = v.x * s - (float)h0, d1 = v.y * s - (float)h1;
             n2 += v.x * v.x + v.y * v.y;
             r2 += d0 * d0 + d1 * d1;
             *reinterpret_cast<ushort2*>(o + c) = make_ushort2(__builtin_bit_cast(unsigned short, h0),
@@ -594,8 +595,8 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(const float* x, int64_
 __global__ __launch_bounds__(256) void screen_codes_kernel(const uint8_t* codes, int64_t rows,
                                                            int dim, int ds, int m, int ks,
                                                            const float* books, float s,
-                                                           float inv_s, unsigned short* out,
-                                                           float* norms, int* max2) {
+                                                           unsigned short* out, float* norms,
+                                                           int* max2) {
     __shared__ float wn[4], wr[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, dsub = dim / m;
     float n_max = 0.f, r_max = 0.f;
@@ -609,7 +610,7 @@ __global__ __launch_bounds__(256) void screen_codes_kernel(const uint8_t* codes,
                 v = books[((int64_t)sub * ks + cr[sub]) * dsub + (c - sub * dsub)];
             }
             const _Float16 hv = to_screen(v, s);
-            const float d = v - (float)hv * inv_s;
+            const float d = v * s - (float)hv;
             n2 += v * v;
             r2 += d * d;
             out[r * ds + c] = __builtin_bit_cast(unsigned short, hv);
@@ -668,7 +669,10 @@ __global__ __launch_bounds__(256) void screen_spread_kernel(const unsigned short
 //   L2: 2 (||q|| dX + dq (X + dX))  +  2 * 2 D u (X^2 / 2 + ||q|| X)  (the scan)
 //       + D u X^2  (the norms)  +  R u (||q|| + X)^2  (the reference's own sums, R terms)
 //   IP: ||q|| dX + dq (X + dX)  +  2 D u ||q|| X  +  R u ||q|| X
-// with 1% on top for the rounding of these figures and of key + err. Where the scales of rows
+// with 1% on top for the rounding of these figures and of key + err. ||q|| and dq are summed of
+// the scaled query, whose largest magnitude is about 2^9: what fp32 loses of its squares (values
+// below 2^-75) is far within the terms in u (of queries near 2^-60 as they are, the squared
+// residuals were all zero, and the nearest row could be ruled out). Where the scales of rows
 // and queries are too far apart for one product to carry both, or a figure overflows, err is
 // +inf, which no query finishes with. Workgroup 0 writes scale: 2^(ex + eq) and its inverse.
 struct QueryScale {
@@ -715,8 +719,9 @@ __global__ __launch_bounds__(256) void screen_queries_kernel(ScreenQueryArgs a) 
             *reinterpret_cast<float2*>(a.padded + q * a.dp + c) = float2{v0, v1};
         const _Float16 h0 = qs.ok ? to_screen(v0, qs.s) : (_Float16)0.f;
         const _Float16 h1 = qs.ok ? to_screen(v1, qs.s) : (_Float16)0.f;
-        const float d0 = v0 - (float)h0 * qs.inv_s, d1 = v1 - (float)h1 * qs.inv_s;
-        n2 += v0 * v0 + v1 * v1;
+        const float w0 = v0 * qs.s, w1 = v1 * qs.s;
+        const float d0 = w0 - (float)h0, d1 = w1 - (float)h1;
+        n2 += w0 * w0 + w1 * w1;
         r2 += d0 * d0 + d1 * d1;
         auto rounds = [](float w) {
             return !((float)(_Float16)w == w && (w == 0.f || fabsf(w) >= 0x1p-14f));
@@ -732,7 +737,7 @@ __global__ __launch_bounds__(256) void screen_queries_kernel(ScreenQueryArgs a) 
     r2 = wave_sum(r2);
     if (lane == 0) {
         const float u = 0x1p-24f, D = (float)a.ds, X = a.x_norm, dX = a.x_res;
-        const float qn = sqrtf(n2), dq = sqrtf(r2);
+        const float qn = sqrtf(n2) * qs.inv_s, dq = sqrtf(r2) * qs.inv_s;
         const float rep = qn * dX + dq * (X + dX), ref = a.ref_terms * u;
         const float e = a.metric == 0 ? 2.f * rep + 4.f * D * u * (0.5f * X * X + qn * X) +
                                             D * u * X * X + ref * (qn + X) * (qn + X)
@@ -1025,7 +1030,7 @@ hipError_t launch_screen_rows(const float* x, int64_t rows, int dp, int ds, int 
     if (rows <= 0) return hipSuccess;
     const int64_t blocks = std::min<int64_t>((rows + 3) / 4, 8192);
     hipLaunchKernelGGL(screen_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, rows, dp,
-                       ds, ldexpf(1.f, e), ldexpf(1.f, -e), out, max2);
+                       ds, ldexpf(1.f, e), out, max2);
     return hipGetLastError();
 }
 
@@ -1035,7 +1040,7 @@ hipError_t launch_screen_codes(const uint8_t* codes, int64_t rows, int dim, int 
     if (rows <= 0) return hipSuccess;
     const int64_t blocks = std::min<int64_t>((rows + 3) / 4, 8192);
     hipLaunchKernelGGL(screen_codes_kernel, dim3((unsigned)blocks), dim3(256), 0, s, codes, rows,
-                       dim, ds, m, ks, books, ldexpf(1.f, e), ldexpf(1.f, -e), out, norms, max2);
+                       dim, ds, m, ks, books, ldexpf(1.f, e), out, norms, max2);
     return hipGetLastError();
 }
 

@@ -177,6 +177,30 @@ def test_magnitudes(gpu):
     assert not _search(idx, q, 10)[2]["screened"]
 
 
+def test_queries_whose_residuals_square_to_nothing(gpu):
+    # Inner products of tiny queries: every rounding residual is about 2^-75, whose square is
+    # no fp32 number, while the largest element, 2^-60, is exact. For each query two rows whose
+    # fp16 keys differ by 0.3 (in units of 2^-89; the other terms of the bound are 0.05) in
+    # favour of one and whose keys differ by 0.5 in favour of the other, 60 residuals of 0.9 / 64
+    # all pulling one way: a bound without the residuals drops the nearest row.
+    rng = np.random.default_rng(975)
+    n, dim, nq = 20_000, 64, 5
+    data = rng.choice([-1, 0, 1], size=(n, dim)).astype(np.float32) * np.float32(2.0 ** -5)
+    data[:, 63] = 0
+    up, down, gap, big = slice(0, 30), slice(30, 60), 60, 63
+    q = np.zeros((nq, dim))
+    q[:, up], q[:, down], q[:, gap], q[:, big] = 40 + 0.9 / 64, 40 - 0.9 / 64, 0.3125, 512
+    for i in range(nq):
+        sign = rng.choice([-1, 1], size=dim)
+        q[i] *= sign
+        data[100 + i] = data[7000 + i] = 0
+        data[100 + i, up] = sign[up]
+        data[7000 + i, down] = sign[down]
+        data[7000 + i, gap] = sign[gap]
+    q = np.ldexp(q, -69).astype(np.float32)
+    _exact(np.ldexp(data, -20), q, 1, oracle.IP)
+
+
 def test_give_up(gpu):
     # a stage wait that gives up (one poll) fails the search; the next one is right
     data, q = datagen.gaussian(200_000, 128, 981), datagen.gaussian(100, 128, 982)
