@@ -32,6 +32,10 @@ int32_t max_magnitude_bits(const float* x, int64_t len);
 bool f16_exact_values(const float* x, int64_t len);
 // SplitMix64 below(n) (pq.rs:34-36) from *state, advancing it.
 uint64_t splitmix_below(uint64_t* state, uint64_t n);
+// Most roundings that a term of a key over n values passes in the reference's arithmetic
+// (distance.rs:3-39): three of the squared difference (an inner product has one), its lane's
+// sum over n / 8 chunks, the eight lanes' sum, and the n % 8 values added one by one.
+inline int64_t ref_roundings(int64_t n) { return 3 + n / 8 + 8 + n % 8; }
 int host_threads();
 // body(lo, hi) over [0, n) in one piece a host thread; where no more threads can be had, the
 // calling one does the rest.
