@@ -36,6 +36,17 @@ uint64_t splitmix_below(uint64_t* state, uint64_t n);
 // (distance.rs:3-39): three of the squared difference (an inner product has one), its lane's
 // sum over n / 8 chunks, the eight lanes' sum, and the n % 8 values added one by one.
 inline int64_t ref_roundings(int64_t n) { return 3 + n / 8 + 8 + n % 8; }
+// A screening scan's fp16 queries: values of all slots (a multiple of a wave's 64), and of the
+// workgroup that its last fragment offsets may lie in, within 32-bit byte offsets.
+constexpr int64_t kScreenBlockSlots = 512;
+inline bool screen_batch_fits(int64_t nq, int64_t ds) {
+    return ((nq + 63) / 64 * 64 + kScreenBlockSlots) * ds <= INT32_MAX / 2;
+}
+// The most queries (at most `most`) of ds padded dims that one screening scan takes; 0: none.
+inline int64_t screen_batch(int64_t ds, int64_t most) {
+    const int64_t slots = (INT32_MAX / 2 / ds - kScreenBlockSlots) / 64 * 64;
+    return std::max<int64_t>(0, std::min(most, slots));
+}
 int host_threads();
 // body(lo, hi) over [0, n) in one piece a host thread; where no more threads can be had, the
 // calling one does the rest.

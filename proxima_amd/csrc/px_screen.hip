@@ -29,6 +29,7 @@
 //   200k of 2M x 384 filtered, 4,096 queries, k = 100 0.68 (930 TFLOP/s)     before 5.38
 //   500k x 100 (128 padded), 4,999 queries, k = 100   0.67                   before 4.95
 #include "px_device.h"
+#include "px_host.h"
 #include "px_kernels.h"
 #include "px_scan_common.h"
 
@@ -45,6 +46,7 @@ namespace {
 
 constexpr int kWaves = 8;
 constexpr int kSlots = 64 * kWaves;            // query slots a workgroup (QB = 2)
+static_assert(kSlots == kScreenBlockSlots, "screen_batch's slots");
 constexpr int kTile = 32;                      // rows a tile: one MFMA block
 constexpr int kTiles = kScreenRows / kTile;    // tiles a row group (4)
 constexpr int kRowBytes = kChunk * 2;          // a staged chunk of a row: 128 fp16
@@ -1000,7 +1002,7 @@ hipError_t launch_flat_screen(const ScreenArgs& a0, hipStream_t s) {
     if (a.spin_limit <= 0) a.spin_limit = kSpinLimit;
     const bool min = a.minima != nullptr;
     if (a.nq <= 0 || a.splits <= 0 || a.rows_per_split % kScreenRows != 0 || !a.spin_fail ||
-        a.ds != a.chunks * kChunk || a.stride < 1 || (screen_query_slots(a.nq) + kSlots) * a.ds > INT32_MAX / 2 ||
+        a.ds != a.chunks * kChunk || a.stride < 1 || !screen_batch_fits(a.nq, a.ds) ||
         (int64_t)a.splits * a.rows_per_split < a.n_eff ||
         (int64_t)(a.splits - 1) * a.rows_per_split >= a.n_eff)
         return hipErrorInvalidValue;

@@ -13,6 +13,8 @@ SHIM = r"""
 #include "px_host.h"
 extern "C" {
 int64_t ref_roundings(int64_t n) { return px::ref_roundings(n); }
+int64_t screen_batch(int64_t ds, int64_t most) { return px::screen_batch(ds, most); }
+int screen_batch_fits(int64_t nq, int64_t ds) { return px::screen_batch_fits(nq, ds); }
 }
 """
 
@@ -27,6 +29,9 @@ def lib(tmp_path_factory):
     lib = ctypes.CDLL(str(out))
     lib.ref_roundings.restype = ctypes.c_int64
     lib.ref_roundings.argtypes = [ctypes.c_int64]
+    lib.screen_batch.restype = ctypes.c_int64
+    for f in (lib.screen_batch, lib.screen_batch_fits):
+        f.argtypes = [ctypes.c_int64, ctypes.c_int64]
     return lib
 
 
@@ -59,3 +64,22 @@ def test_ref_roundings_cover_every_width(lib):
         for m in (1, 2, 7, 48):
             entry = _roundings(dsub, 3)
             assert lib.ref_roundings(dsub) + m >= entry + m - 1, (dsub, m)
+
+
+def test_screen_batch_is_what_the_scan_takes(lib):
+    # every batch that a screened search is cut into is one the scan's launcher accepts: past
+    # 63,500 dims it is fewer than 16,384 queries, past 1.8M none (such searches are not screened)
+    seen = set()
+    for ds in [128, 384, 1024, 16_384, 63_488, 63_616, 65_536, 233_088, 1_000_064, 1_863_936,
+               1_864_192, 1_900_032, 3_000_064, 2 ** 31]:
+        b = lib.screen_batch(ds, 16_384)
+        seen.add(b)
+        assert 0 <= b <= 16_384
+        if b:
+            assert lib.screen_batch_fits(b, ds)
+        if b < 16_384:
+            assert not lib.screen_batch_fits(b + 64, ds), (ds, b)
+        assert lib.screen_batch(ds, 1) == min(b, 1)
+        assert lib.screen_batch(ds, 1000) == min(b, 1000)
+    assert 0 in seen and 16_384 in seen and len(seen) > 4
+    assert not lib.screen_batch_fits(16_384, 63_616)  # one launch of the whole batch is refused
