@@ -7,6 +7,7 @@ Python surface raises). Each failure must leave the index as it was -- rows coun
 unchanged -- and the same index must work again once memory is there.
 """
 import contextlib
+import gc
 import os
 
 import numpy as np
@@ -80,3 +81,45 @@ def test_pq_train_and_add_out_of_memory(gpu):
     ids, d = pq.search_batch(q, k=10)
     o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), pq.codes(), q, 10, oracle.L2)
     assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
+
+
+def test_flat_add_that_fits_without_the_screening_copy(gpu):
+    # 40,000 rows of 128 dims: 20.5 MB and a screening copy of 10.2; the next row grows the index
+    # to 80,000 rows' room, 41 MB beside the old rows. 67 MB hold both and a search's scratch, not
+    # the copy too: the copy gives way, and is made again (20.5 MB) once the old rows are gone.
+    gc.collect()
+    data = datagen.gaussian(40_001, 128, 321)
+    q = datagen.gaussian(30, 128, 322)
+    idx = FlatIndex(128, Metric.L2)
+    idx.add(data[:40_000])
+    idx.search_batch(q, k=10)
+    assert idx._last_timing()["screened"]
+    print("case flat add that fits without the copy", flush=True)
+    with device_budget(67_000_000):
+        idx.add(data[40_000:])
+        ids, d = idx.search_batch(q, k=10)
+    assert idx._last_timing()["screened"]
+    o_ids, o_d, _ = oracle.flat_search(data, q, 10, oracle.L2)
+    assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
+
+
+def test_pq_add_that_fits_without_the_screening_copy(gpu):
+    # 100,000 codes of 64 bytes: 6.4 MB and a copy of 26; room for twice as many is 12.8 MB more,
+    # which 40 MB hold without the copy (and not the 51 MB copy after)
+    gc.collect()
+    rng = np.random.default_rng(323)
+    pq = PqIndex(64, Metric.L2, m=64, train_iters=1, train_sample=1000)
+    pq.train(datagen.gaussian(1000, 64, 324))
+    codes = rng.integers(0, 256, size=(100_001, 64)).astype(np.uint8)
+    pq.add_codes(codes[:100_000])
+    q = datagen.gaussian(20, 64, 325)
+    pq.search_batch(q, k=10)
+    assert pq._last_timing()["screened"]
+    print("case pq add that fits without the copy", flush=True)
+    with device_budget(40_000_000):
+        pq.add_codes(codes[100_000:])
+        ids, d = pq.search_batch(q, k=10)
+        assert not pq._last_timing()["screened"]
+    o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), codes, q, 10, oracle.L2)
+    assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
+    pq.search_batch(q, k=10)
