@@ -123,3 +123,42 @@ def test_pq_add_that_fits_without_the_screening_copy(gpu):
     o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), codes, q, 10, oracle.L2)
     assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
     pq.search_batch(q, k=10)
+
+
+@pytest.mark.parametrize("budget,copy_kept", [(78_700_000, True), (77_400_000, False)])
+def test_flat_search_that_fits_without_screening(gpu, budget, copy_kept):
+    # 100,000 rows of 128 dims and their copy: 77.2 MB. A screened search of 17 queries wants 2.3
+    # MB of candidates, the fp32 lists 0.6: 78.7 MB hold those, 77.4 only without the copy.
+    gc.collect()
+    data = datagen.gaussian(100_000, 128, 331)
+    q = datagen.gaussian(17, 128, 332)
+    idx = FlatIndex(128, Metric.L2)
+    idx.add(data)
+    o_ids, o_d, _ = oracle.flat_search(data, q, 10, oracle.L2)
+    print(f"case flat search without screening, budget {budget}", flush=True)
+    with device_budget(budget):
+        ids, d = idx.search_batch(q, k=10)
+        assert not idx._last_timing()["screened"]
+        assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
+    ids, d = idx.search_batch(q, k=10)
+    assert idx._last_timing()["screened"] == copy_kept
+    assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
+    idx.add(data[:1])  # (room for it: the copy is brought up to date, or made again)
+    idx.search_batch(q, k=10)
+    assert idx._last_timing()["screened"]
+
+
+def test_pq_search_that_fits_without_screening(gpu):
+    # 100,000 codes of 16 bytes of 32 dims: 1.6 MB and a copy of 26; 500 queries, k = 10
+    gc.collect()
+    data = datagen.gaussian(100_000, 32, 341)
+    q = datagen.gaussian(500, 32, 342)
+    pq = PqIndex(32, Metric.L2, m=16, train_iters=1, train_sample=1000)
+    pq.train(data)
+    pq.add(data)
+    print("case pq search without screening", flush=True)
+    with device_budget(29_500_000):
+        ids, d = pq.search_batch(q, k=10)
+        assert not pq._last_timing()["screened"]
+    o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), pq.codes(), q, 10, oracle.L2)
+    assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
