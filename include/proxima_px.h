@@ -192,23 +192,24 @@ int px_hip_versions(int* runtime_version, int* driver_version);
 int px_flat_set_timing(px_flat* idx, int enable);
 int px_flat_last_timing(const px_flat* idx, float* scan_ms, float* total_ms, int* splits,
                         int* blocks);
-/* Collect rounds of the handle's last search: 0 when it used per-split candidate lists (or
- * the screening scan in their place, finished in its one round), else the rounds of the
- * threshold-collect path (1 when every query finished in the first). Diagnostic; no
- * counterpart in the reference. */
+/* Collect rounds of the handle's last search: 0 when it used per-split candidate lists, else
+ * the rounds of the threshold-collect path (1 when every query finished in the first) or, of
+ * a screened search, its own rounds and those of the path that finished what it left open.
+ * Diagnostic; no counterpart in the reference. */
 int px_flat_last_rounds(const px_flat* idx, int* rounds);
 /* Selection path of the handle's last search: PX_PATH_LISTS (per-split candidate lists),
  * PX_PATH_COLLECT_SAMPLED (threshold-collect whose first round takes its thresholds from a
  * strided row sample), PX_PATH_COLLECT_BOUNDED (threshold-collect whose first round is
  * bounded by the splits' shared bound alone, no sample), PX_PATH_VECTOR (the vector-ALU
- * collect scan of a few queries), PX_PATH_FULL_SORT (k past PX_MAX_K). A screened search
- * (px_flat_last_screened) reports the path whose scan the screening scan stands in for.
- * Diagnostic; no counterpart in the reference. */
+ * collect scan of a few queries), PX_PATH_FULL_SORT (k past PX_MAX_K), PX_PATH_SCREENED (the
+ * screening scan, px_flat_set_screening; queries it left open went through one of the
+ * others). Diagnostic; no counterpart in the reference. */
 #define PX_PATH_LISTS 0
 #define PX_PATH_COLLECT_SAMPLED 1
 #define PX_PATH_COLLECT_BOUNDED 2
 #define PX_PATH_VECTOR 3
 #define PX_PATH_FULL_SORT 4 /* k past PX_MAX_K: every key computed and sorted */
+#define PX_PATH_SCREENED 5
 int px_flat_last_path(const px_flat* idx, int* path);
 /* Use of the fp16 copy of 128-dim rows. The copy (2 bytes a value) is kept from the first
  * px_flat_add while every row added is exactly an fp16 zero or normal number (integer-valued
@@ -217,15 +218,20 @@ int px_flat_last_path(const px_flat* idx, int* path);
  * list scan on at least 65,536 rows (each product is exact in fp16 as in fp32; the
  * candidates are re-ranked in the reference's arithmetic as on fp32), and the vector-ALU
  * scan of batches of at most 16 queries reads the copy and widens it to the same fp32
- * values. enable = 0 keeps both scans on the fp32 rows (default 1). Diagnostic and
- * tuning; no counterpart in the reference. */
+ * values. enable = 0 keeps both scans on the fp32 rows and turns screening off
+ * (px_flat_set_screening; default 1). Diagnostic and tuning; no counterpart in the
+ * reference. */
 int px_flat_set_scan_f16(px_flat* idx, int enable);
-/* *used = 1 if the handle's last search read the fp16 copy of the rows (either scan), else
- * 0. */
+/* *used = 1 if the handle's last search ran one of those scans on the fp16 copy of the rows,
+ * else 0. */
 int px_flat_last_scan_f16(const px_flat* idx, int* used);
-/* *used = 1 if the handle's last search was screened: its fp32 scan replaced by one of the
- * rows rounded to fp16, which rules out only rows proven not to be among the results
- * (results unchanged; px_flat_set_scan_f16(idx, 0) turns it off), else 0. */
+/* Screening of searches: the scan of the fp32 rows replaced by one of a copy of them rounded to
+ * fp16, which rules out only rows proven not to be among the results; the keys of the rest are
+ * computed in the reference's arithmetic. The copy takes 2 bytes a value, dims rounded up to
+ * whole 128s, beside the rows (rows with the fp16 copy above need no other). enable = 0 frees
+ * the copy, keeps none and searches without (default 1). No counterpart in the reference. */
+int px_flat_set_screening(px_flat* idx, int enable);
+/* *used = 1 if the handle's last search was screened, else 0. */
 int px_flat_last_screened(const px_flat* idx, int* used);
 /* Polls a stage-sync wait of the barrier-free scans (the collect scans; lists of k + 8 <= 32)
  * makes before it gives up; 0 (the default) keeps the kernels' own, 2^16 polls, about 5 ms.
@@ -234,9 +240,12 @@ int px_flat_last_screened(const px_flat* idx, int* used);
  * unwritten. A handle's later searches are unaffected. Test hook (a small limit forces the
  * give-up); no counterpart in the reference. */
 int px_flat_set_spin_limit(px_flat* idx, int polls);
-/* The same for PqIndex searches (k <= 128: per-wave lists; above: threshold-collect). */
+/* The same as px_flat_last_rounds for PqIndex searches (k <= 128: per-wave lists; above:
+ * threshold-collect; screened searches as there). */
 int px_pq_last_rounds(const px_pq* idx, int* rounds);
-/* As px_flat_last_screened. */
+/* As px_flat_set_screening and px_flat_last_screened; the copy is of the rows that the codes
+ * stand for, at most 8 GiB. Off, every search runs the scan on lookup tables. */
+int px_pq_set_screening(px_pq* idx, int enable);
 int px_pq_last_screened(const px_pq* idx, int* used);
 int px_pq_set_timing(px_pq* idx, int enable);
 int px_pq_last_timing(const px_pq* idx, float* scan_ms, float* total_ms, int* splits,

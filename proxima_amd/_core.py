@@ -269,8 +269,13 @@ class FlatIndex:
     def _scan_f16(self, enable: bool = True) -> None:
         """Use the fp16 copy of rows exact in fp16 (default on): the collect scan multiplies
         in fp16 where the queries are exact too, the few-query vector scan reads the copy;
-        off keeps both on the fp32 rows. Diagnostic; no counterpart in the reference."""
+        off keeps both on the fp32 rows and turns screening off. Diagnostic; no counterpart in the reference."""
         _check(self._lib.px_flat_set_scan_f16(self._h, 1 if enable else 0))
+
+    def _screening(self, enable: bool = True) -> None:
+        """Screen searches on an fp16 copy of the rows (default on); off frees the copy and
+        searches with the other scans. No counterpart in the reference."""
+        _check(self._lib.px_flat_set_screening(self._h, 1 if enable else 0))
 
     def _spin_limit(self, polls: int = 0) -> None:
         """Polls a stage-sync wait of the barrier-free scans makes before it gives up (0: the
@@ -291,7 +296,7 @@ class FlatIndex:
         return {"scan_ms": scan.value, "total_ms": total.value, "splits": splits.value,
                 "blocks": blocks.value, "collect_rounds": rounds.value,
                 "path": ("lists", "collect-sampled", "collect-bounded", "vector",
-                         "full-sort")[path.value],
+                         "full-sort", "screened")[path.value],
                 "scan_f16": bool(f16.value), "screened": bool(screened.value)}
 
 
@@ -500,6 +505,11 @@ class PqIndex:
         if n:
             idx.add_codes(codes.reshape(n, m))
         return idx
+
+    def _screening(self, enable: bool = True) -> None:
+        """Screen searches on an fp16 copy of the decoded rows (default on); off frees the copy
+        and searches with lookup tables. No counterpart in the reference."""
+        _check(self._lib.px_pq_set_screening(self._h, 1 if enable else 0))
 
     def _timing(self, enable: bool = True) -> None:
         _check(self._lib.px_pq_set_timing(self._h, 1 if enable else 0))

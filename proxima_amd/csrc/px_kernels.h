@@ -201,7 +201,7 @@ struct ScreenQueryArgs {
     float* padded;             // optional, out: the queries [nq][dp], zero pad columns
     // optional, two ints: [0] = 0 (ScreenArgs::spin_fail), [1]: with parts (whose launch
     // cleared both), 1 if a query holds a NaN or an infinite value (every err is infinite
-    // then), 2 if a value is not exactly an fp16 zero or normal number; without, 0
+    // then); without, 0
     int* words;
     unsigned short* qs;        // out: ScreenArgs::qs
     float* err;                // out, by query: bound on |scan key - reference key|

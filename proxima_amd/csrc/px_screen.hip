@@ -702,7 +702,7 @@ __global__ __launch_bounds__(256) void screen_queries_kernel(ScreenQueryArgs a) 
         a.scale[1] = ldexpf(1.f, -(a.ex + qs.eq));
         if (a.words) {
             if (!a.parts) a.words[0] = a.words[1] = 0;
-            else if (m > FLT_MAX) atomicOr(a.words + 1, 1);
+            else if (m > FLT_MAX) a.words[1] = 1;
         }
     }
     // slot sl holds query q; padding slots are zeros
@@ -713,7 +713,6 @@ __global__ __launch_bounds__(256) void screen_queries_kernel(ScreenQueryArgs a) 
     const float* x = a.queries + q * a.pitch;
     unsigned short* o = a.qs + (sl >> 5) * 32 * a.ds + (sl & 31) * 8;
     float n2 = 0.f, r2 = 0.f;
-    bool inexact = false;
     for (int c = lane * 2; c < a.ds; c += 128) {
         const float v0 = live && c < a.dim ? x[c] : 0.f;
         const float v1 = live && c + 1 < a.dim ? x[c + 1] : 0.f;
@@ -725,16 +724,11 @@ __global__ __launch_bounds__(256) void screen_queries_kernel(ScreenQueryArgs a) 
         const float d0 = w0 - (float)h0, d1 = w1 - (float)h1;
         n2 += w0 * w0 + w1 * w1;
         r2 += d0 * d0 + d1 * d1;
-        auto rounds = [](float w) {
-            return !((float)(_Float16)w == w && (w == 0.f || fabsf(w) >= 0x1p-14f));
-        };
-        inexact |= rounds(v0) || rounds(v1);
         // fragment order: 16-dim group c / 16, half (c / 8) % 2, query, dim c % 8
         *reinterpret_cast<ushort2*>(o + (c >> 3) * 256 + (c & 7)) = make_ushort2(
             __builtin_bit_cast(unsigned short, h0), __builtin_bit_cast(unsigned short, h1));
     }
     if (!live) return;
-    if (a.words && a.parts && __ballot(inexact) && lane == 0) atomicOr(a.words + 1, 2);
     n2 = wave_sum(n2);
     r2 = wave_sum(r2);
     if (lane == 0) {

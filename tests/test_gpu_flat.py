@@ -28,11 +28,18 @@ def _run(data, queries, k, metric, mask=None):
     m = Metric.L2 if metric == oracle.L2 else Metric.InnerProduct
     idx = FlatIndex(data.shape[1], m)
     idx.add(data)
-    if mask is None:
-        ids, d = idx.search_batch(queries, k=k)
-    else:
-        ids, d = idx.search_batch_filtered(queries, mask, k=k)
     o_ids, o_d, _ = oracle.flat_search(data, queries, k, metric, mask=mask)
+    # as every program searches, checked here; then on the scans that screening stands in for,
+    # which these tests are about
+    for screening in (True, False):
+        idx._screening(screening)
+        if mask is None:
+            ids, d = idx.search_batch(queries, k=k)
+        else:
+            ids, d = idx.search_batch_filtered(queries, mask, k=k)
+        if screening:
+            assert_parity(ids, d, o_ids, o_d, _oracle_key(data, queries, metric))
+    assert not idx._last_timing()["screened"]
     return ids, d, o_ids, o_d
 
 
@@ -294,6 +301,8 @@ def test_device_pointer_entry(gpu):
     (2048, 10, False, "collect-bounded"),
     (300, 200, False, "collect-sampled"),
     (5, 10, False, "vector"),
+    (200, 10, False, "screened"),
+    (5, 10, True, "screened"),
 ])
 def test_device_query_nonfinite_leaves_outputs(gpu, nq, k, masked, path):
     # flat.rs:114-117 rejects a NaN or infinite query before searching: the device form
@@ -305,6 +314,7 @@ def test_device_query_nonfinite_leaves_outputs(gpu, nq, k, masked, path):
     mask = datagen.mask(40_000, 0.5, 46) if masked else None
     idx = FlatIndex(64, Metric.L2)
     idx.add(data)
+    idx._screening(path == "screened")
     ptrs = []
 
     def dev(arr):

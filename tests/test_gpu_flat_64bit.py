@@ -6,7 +6,8 @@ starts beyond a 32-bit element offset. The reference indexes rows with usize
 tile loads, the row ids of a filter and the exact re-rank must all address past 2^31
 elements. Each path that a search can take on these rows runs once: the MFMA collect scan
 with several query chunks, unfiltered and filtered (k = 100, 300 queries), the per-split
-lists (k = 10, 64 queries) and the vector-ALU scan (k = 10, 8 queries). Queries 0-19 are
+lists (k = 10, 64 queries) and the vector-ALU scan (k = 10, 8 queries), each with screening
+off, and the same searches on the screening scan. Queries 0-19 are
 copies of rows past the boundary, so that their nearest rows lie there; a sample of the
 queries (the oracle scans 8.6 GB per query) is checked against the oracle at the parity
 rule.
@@ -43,46 +44,41 @@ def _key_of(data, queries):
     return lambda qi, row: -float(oracle.inner_product(queries[qi], data[row]))
 
 
-def _check(data, q, ids, d, sample, k, mask=None):
+def _check(big, nq, sample, k, paths, mask=None):
+    """The first nq queries on the scan of `paths` and on the screening scan: the planted rows
+    first, `sample` of the queries against the oracle."""
+    data, q, planted_rows, idx = big
+    q = q[:nq]
+    planted = min(nq, PLANTED)
     o_ids, o_d, _ = oracle.flat_search(data, q[sample], k, oracle.IP, mask=mask)
-    assert_parity(ids[sample], d[sample], o_ids, o_d, _key_of(data, q[sample]))
+    for path in (paths, ("screened",)):
+        print(f"case: {nq} queries, k={k}, mask={mask is not None}, {path}", flush=True)
+        idx._screening(path == ("screened",))
+        ids, d = (idx.search_batch(q, k=k) if mask is None
+                  else idx.search_batch_filtered(q, mask, k=k))
+        assert idx._last_timing()["path"] in path
+        assert np.array_equal(ids[:planted, 0], planted_rows[:planted])
+        assert_parity(ids[sample], d[sample], o_ids, o_d, _key_of(data, q[sample]))
+    return ids
 
 
 def test_collect_scan_past_2_31_elements(big):
-    data, q, planted_rows, idx = big
-    print("case: 300 queries, k=100, unfiltered (collect scan, 3 query chunks)", flush=True)
-    ids, d = idx.search_batch(q, k=100)
-    assert idx._last_timing()["path"] in ("collect-sampled", "collect-bounded")
-    assert np.array_equal(ids[:PLANTED, 0], planted_rows)
+    # 3 query chunks
+    ids = _check(big, 300, np.r_[0:8, 23:300:12], 100, ("collect-sampled", "collect-bounded"))
     assert (ids >= BOUNDARY).sum() > PLANTED
-    _check(data, q, ids, d, np.r_[0:8, 23:300:12], 100)
 
 
 def test_filtered_collect_scan_past_2_31_elements(big):
-    data, q, planted_rows, idx = big
     mask = datagen.config_mask(5, n=ROWS)
-    mask[planted_rows] = True
-    print("case: 300 queries, k=100, 10% filter (filtered collect scan)", flush=True)
-    ids, d = idx.search_batch_filtered(q, mask, k=100)
-    assert idx._last_timing()["path"] in ("collect-sampled", "collect-bounded")
-    assert np.array_equal(ids[:PLANTED, 0], planted_rows)
+    mask[big[2]] = True
+    ids = _check(big, 300, np.r_[0:8, 29:300:12], 100, ("collect-sampled", "collect-bounded"),
+                 mask=mask)
     assert mask[ids[ids >= 0]].all()
-    _check(data, q, ids, d, np.r_[0:8, 29:300:12], 100, mask=mask)
 
 
 def test_lists_past_2_31_elements(big):
-    data, q, planted_rows, idx = big
-    print("case: 64 queries, k=10 (per-split lists)", flush=True)
-    ids, d = idx.search_batch(q[:64], k=10)
-    assert idx._last_timing()["path"] == "lists"
-    assert np.array_equal(ids[:PLANTED, 0], planted_rows)
-    _check(data, q[:64], ids, d, np.r_[0:64:2], 10)
+    _check(big, 64, np.r_[0:64:2], 10, ("lists",))
 
 
 def test_vector_scan_past_2_31_elements(big):
-    data, q, planted_rows, idx = big
-    print("case: 8 queries, k=10 (vector-ALU scan)", flush=True)
-    ids, d = idx.search_batch(q[:8], k=10)
-    assert idx._last_timing()["path"] == "vector"
-    assert np.array_equal(ids[:, 0], planted_rows[:8])
-    _check(data, q[:8], ids, d, np.arange(8), 10)
+    _check(big, 8, np.arange(8), 10, ("vector",))

@@ -40,8 +40,10 @@ def _rounds(idx) -> int:
     return r.value
 
 
-def _search(data, queries, k, metric, mask=None):
+def _search(data, queries, k, metric, mask=None, screening=False):
+    """One search without screening (unless said), whose scans these tests are about."""
     idx = FlatIndex(data.shape[1], Metric.L2 if metric == oracle.L2 else Metric.InnerProduct)
+    idx._screening(screening)
     idx.add(data)
     if mask is None:
         ids, d = idx.search_batch(queries, k=k)
@@ -53,12 +55,14 @@ def _search(data, queries, k, metric, mask=None):
 def _check(data, queries, k, metric, mask=None, exact=False):
     print(f"case n={data.shape[0]} dim={data.shape[1]} nq={queries.shape[0]} k={k} "
           f"metric={metric} mask={'yes' if mask is not None else 'no'}", flush=True)
-    idx, ids, d = _search(data, queries, k, metric, mask)
     o_ids, o_d, _ = oracle.flat_search(data, queries, k, metric, mask=mask)
-    assert_parity(ids, d, o_ids, o_d, _key_of(data, queries, metric), allow_exempt=not exact)
-    if exact:
-        assert np.array_equal(ids, o_ids)
-        assert np.array_equal(d.view(np.uint32), o_d.view(np.uint32))
+    for screening in (True, False):
+        idx, ids, d = _search(data, queries, k, metric, mask, screening)
+        assert_parity(ids, d, o_ids, o_d, _key_of(data, queries, metric), allow_exempt=not exact)
+        if exact:
+            assert np.array_equal(ids, o_ids)
+            assert np.array_equal(d.view(np.uint32), o_d.view(np.uint32))
+    assert not idx._last_timing()["screened"]
     return _rounds(idx)
 
 
@@ -253,6 +257,7 @@ def test_sample_short_of_its_last_split(gpu):
     k = 100
     print(f"case n=10000 dim=128 nq=300 k={k} L2, twice", flush=True)
     idx = FlatIndex(128, Metric.L2)
+    idx._screening(False)
     idx.add(data)
     o_ids, o_d, _ = oracle.flat_search(data, q, k, oracle.L2)
     for _ in range(2):
@@ -380,6 +385,7 @@ data = rng.integers(0, 4, size=(n, {dim})).astype(np.float32)
 data[np.arange(s) * n // s] = 255.0  # the sampled positions, floor(i * n / s)
 q = rng.integers(0, 3, size=(300, {dim})).astype(np.float32)
 idx = FlatIndex({dim}, Metric.L2)
+idx._screening(False)
 idx.add(data)
 ids, d = idx.search_batch(q, k=k)
 o_ids, o_d, _ = oracle.flat_search(data, q, k, oracle.L2)
@@ -476,6 +482,7 @@ def test_bound_only_consecutive_searches(gpu):
     qa = datagen.sift_like(2048, 64, 71)
     qb = datagen.sift_like(2048, 64, 72) // 4
     idx = FlatIndex(64, Metric.L2)
+    idx._screening(False)
     idx.add(data)
     ref = {}
     for name, q in (("a", qa), ("b", qb)):

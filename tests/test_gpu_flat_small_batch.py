@@ -39,7 +39,10 @@ def _check(data, queries, k, metric, mask=None, exact=False, searches=1):
     idx = FlatIndex(data.shape[1], Metric.L2 if metric == oracle.L2 else Metric.InnerProduct)
     idx.add(data)
     o_ids, o_d, _ = oracle.flat_search(data, queries, k, metric, mask=mask)
-    for _ in range(searches):
+    # once as every program searches (screened, where the sizes are), then on the scan that these
+    # tests are about
+    for screening in [True] + [False] * searches:
+        idx._screening(screening)
         if mask is None:
             ids, d = idx.search_batch(queries, k=k)
         else:
@@ -49,6 +52,7 @@ def _check(data, queries, k, metric, mask=None, exact=False, searches=1):
         if exact:
             assert np.array_equal(ids, o_ids)
             assert np.array_equal(d.view(np.uint32), o_d.view(np.uint32))
+    assert idx._last_timing()["path"] in ("vector", "lists")
     return _rounds(idx)
 
 

@@ -21,6 +21,15 @@ def _index(data, m, nbits, metric, iters=8, sample=0, seed=24301):
     return pq
 
 
+def _both(pq):
+    """Twice through a search: as every program runs it (screened, where the sizes are), then
+    with the scan on lookup tables, which these tests are about."""
+    for screening in (True, False):
+        pq._screening(screening)
+        yield
+        assert screening or not pq._last_timing()["screened"]
+
+
 @pytest.mark.parametrize("m,nbits", [(16, 8), (8, 8), (4, 6), (6, 4), (12, 3)])
 @pytest.mark.parametrize("metric", [oracle.L2, oracle.IP])
 def test_pq_bit_exact(gpu, m, nbits, metric):
@@ -33,11 +42,12 @@ def test_pq_bit_exact(gpu, m, nbits, metric):
     assert np.array_equal(books, oracle.pq_train(data, m, nbits, 8, 0, 24301))
     assert np.array_equal(codes, oracle.pq_encode(books, data))
     for k in (1, 10, 64):
-        ids, d = pq.search_batch(q, k=k)
         o_ids, o_d, _ = oracle.pq_search(books, codes, q, k, metric)
         print(f"pq m={m} nbits={nbits} metric={metric} k={k}", flush=True)
-        assert np.array_equal(ids, o_ids)
-        assert np.array_equal(d, o_d)
+        for _ in _both(pq):
+            ids, d = pq.search_batch(q, k=k)
+            assert np.array_equal(ids, o_ids)
+            assert np.array_equal(d, o_d)
 
 
 @pytest.mark.parametrize("p", [0.0, 0.01, 0.5])
@@ -46,11 +56,12 @@ def test_pq_filtered_bit_exact(gpu, p):
     q = datagen.gaussian(40, 64, 6)
     mask = datagen.mask(20_000, p, 7)
     pq = _index(data, 16, 8, oracle.L2, iters=4, sample=5000)
-    ids, d = pq.search_batch_filtered(q, mask, k=10)
     o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), pq.codes(), q, 10, oracle.L2, mask=mask)
-    assert np.array_equal(ids, o_ids)
-    assert np.array_equal(d, o_d)
-    assert mask[ids[ids >= 0]].all()
+    for _ in _both(pq):
+        ids, d = pq.search_batch_filtered(q, mask, k=10)
+        assert np.array_equal(ids, o_ids)
+        assert np.array_equal(d, o_d)
+        assert mask[ids[ids >= 0]].all()
 
 
 def test_pq_config4_reduced(gpu):
@@ -63,11 +74,12 @@ def test_pq_config4_reduced(gpu):
     pq.add(data)
     books, codes = pq.codebooks(), pq.codes()
     for msk in (None, mask):
-        ids, d = (pq.search_batch(q, k=10) if msk is None else
-                  pq.search_batch_filtered(q, msk, k=10))
         o_ids, o_d, _ = oracle.pq_search(books, codes, q, 10, oracle.L2, mask=msk)
-        assert np.array_equal(ids, o_ids)
-        assert np.array_equal(d, o_d)
+        for _ in _both(pq):
+            ids, d = (pq.search_batch(q, k=10) if msk is None else
+                      pq.search_batch_filtered(q, msk, k=10))
+            assert np.array_equal(ids, o_ids)
+            assert np.array_equal(d, o_d)
 
 
 def test_pq_recall_reference_thresholds(gpu):
@@ -120,10 +132,11 @@ def test_pq_few_queries_many_lists_exact(gpu, nq):
     q = datagen.gaussian(nq, 32, 302)
     pq = _index(data, 8, 8, oracle.L2, iters=4, sample=5000)
     for k in (1, 10, 50):
-        ids, d = pq.search_batch(q, k=k)
         o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), pq.codes(), q, k, oracle.L2)
-        assert np.array_equal(ids, o_ids), k
-        assert np.array_equal(d, o_d), k
+        for _ in _both(pq):
+            ids, d = pq.search_batch(q, k=k)
+            assert np.array_equal(ids, o_ids), k
+            assert np.array_equal(d, o_d), k
 
 
 def test_pq_few_queries_heavy_ties(gpu):
@@ -132,7 +145,8 @@ def test_pq_few_queries_heavy_ties(gpu):
     data = datagen.gaussian(100_000, 8, 303)
     q = datagen.gaussian(2, 8, 304)
     pq = _index(data, 2, 2, oracle.IP, iters=3, sample=2000)
-    ids, d = pq.search_batch(q, k=20)
     o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), pq.codes(), q, 20, oracle.IP)
-    assert np.array_equal(ids, o_ids)
-    assert np.array_equal(d, o_d)
+    for _ in _both(pq):
+        ids, d = pq.search_batch(q, k=20)
+        assert np.array_equal(ids, o_ids)
+        assert np.array_equal(d, o_d)

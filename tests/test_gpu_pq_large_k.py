@@ -36,13 +36,17 @@ def _rounds(pq) -> int:
 def _check(pq, q, k, metric, mask=None):
     print(f"pq case n={len(pq)} nq={q.shape[0]} k={k} metric={metric} "
           f"mask={'yes' if mask is not None else 'no'}", flush=True)
-    if mask is None:
-        ids, d = pq.search_batch(q, k=k)
-    else:
-        ids, d = pq.search_batch_filtered(q, mask, k=k)
     o_ids, o_d, _ = oracle.pq_search(pq.codebooks(), pq.codes(), q, k, metric, mask=mask)
-    assert np.array_equal(ids, o_ids)
-    assert np.array_equal(d, o_d)
+    # as every program searches, then on the lookup tables' scans, which these tests are about
+    for screening in (True, False):
+        pq._screening(screening)
+        if mask is None:
+            ids, d = pq.search_batch(q, k=k)
+        else:
+            ids, d = pq.search_batch_filtered(q, mask, k=k)
+        assert np.array_equal(ids, o_ids)
+        assert np.array_equal(d, o_d)
+    assert not pq._last_timing()["screened"]
     return _rounds(pq)
 
 

@@ -30,7 +30,10 @@ def _key_of(data, queries, metric):
 
 
 def _index(data, metric):
+    """An index whose searches take these scans (and their fp32 forms), not the screening scan
+    that reads the same copy for lists and few queries."""
     idx = FlatIndex(data.shape[1], Metric.L2 if metric == oracle.L2 else Metric.InnerProduct)
+    idx._screening(False)
     idx.add(data)
     return idx
 

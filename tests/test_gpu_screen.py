@@ -39,7 +39,7 @@ def _exact(data, q, k, metric, mask=None, idx=None):
           f"metric={metric} mask={mask is not None}", flush=True)
     idx = idx or _index(data, metric)
     ids, d, info = _search(idx, q, k, mask)
-    assert info["screened"] and not info["scan_f16"], info
+    assert info["screened"] and info["path"] == "screened" and not info["scan_f16"], info
     o_ids, o_d, _ = oracle.flat_search(data, q, k, metric, mask=mask)
     _same((ids, d), (o_ids, o_d))
     return idx, info
@@ -63,7 +63,7 @@ def _exact(data, q, k, metric, mask=None, idx=None):
 def test_sizes(gpu, n, dim, nq, k, metric, kind):
     gen = {"gauss": datagen.gaussian, "unit": datagen.unit_gaussian, "sift": datagen.sift_like}[kind]
     _, info = _exact(gen(n, dim, 901), gen(nq, dim, 902), k, metric)
-    assert info["collect_rounds"] == (0 if info["path"] == "lists" else 1)
+    assert info["collect_rounds"] == 1
 
 
 @pytest.mark.parametrize("dim", [96, 200])
@@ -139,7 +139,7 @@ def test_what_screening_leaves_open(gpu, name):
     # (rows so far from the origin that fp16 cannot tell them apart are not screened)
     assert info["screened"] == (name != "offset")
     if name == "query scale":
-        assert info["collect_rounds"] >= 1  # the fp32 collect scan's
+        assert info["collect_rounds"] >= 2  # and the fp32 collect scan's
     idx._scan_f16(False)
     ids32, d32, info32 = _search(idx, q, 10)
     assert not info32["screened"]
@@ -286,7 +286,7 @@ def test_rows_exact_in_fp16(gpu, nq, k, exact):
         idx = _index(data, metric)
         o = oracle.flat_search(data, q, k, metric)[:2]
         ids, d, info = _search(idx, q, k)
-        assert info["screened"] and info["scan_f16"] == (exact or nq <= 16), info
+        assert info["screened"] and not info["scan_f16"], info
         _same((ids, d), o)
         bufs = [(ctypes.c_void_p(), n) for n in (q.nbytes, nq * k * 8, nq * k * 4)]
         try:
@@ -296,13 +296,67 @@ def test_rows_exact_in_fp16(gpu, nq, k, exact):
             assert lib.px_dev_upload(dq, q.ctypes.data, q.nbytes) == 0
             assert lib.px_flat_search_device(idx._h, dq, nq, k, None, di, dd) == 0
             info = idx._last_timing()
-            assert info["screened"] and info["scan_f16"] == (exact or nq <= 16), info
+            assert info["screened"] and not info["scan_f16"], info
             assert lib.px_dev_download(ids.ctypes.data, di, ids.nbytes) == 0
             assert lib.px_dev_download(d.ctypes.data, dd, d.nbytes) == 0
             _same((ids, d), o)
         finally:
             for p, _ in bufs:
                 lib.px_dev_free(p)
+
+
+def test_what_ran_is_reported(gpu):
+    # a screened search reports the screening scan, its own rounds and no other scan; with
+    # screening off the same search reports the scan that takes its place, and so does the
+    # no-allocation entry point, which is never screened
+    import ctypes
+    from proxima_amd import _lib
+    lib = _lib.load()
+    data, q = datagen.gaussian(30_000, 64, 1001), datagen.gaussian(40, 64, 1002)
+    idx = _index(data, oracle.L2)
+
+    def said():
+        t = idx._last_timing()
+        return [t[x] for x in ("screened", "path", "scan_f16", "collect_rounds")]
+
+    _search(idx, q, 10)
+    assert said() == [True, "screened", False, 1]
+    bufs = [(ctypes.c_void_p(), n) for n in (q.nbytes, 40 * 10 * 8, 40 * 10 * 4)]
+    try:
+        for p, n in bufs:
+            assert lib.px_dev_alloc(ctypes.byref(p), n) == 0
+        (dq, _), (di, _), (dd, _) = bufs
+        assert lib.px_dev_upload(dq, q.ctypes.data, q.nbytes) == 0
+        assert lib.px_flat_search_device_noalloc(idx._h, dq, 40, 10, None, di, dd) == 0
+    finally:
+        for p, _ in bufs:
+            lib.px_dev_free(p)
+    assert said() == [False, "lists", False, 0]
+    idx._screening(False)
+    _search(idx, q, 10)
+    assert said() == [False, "lists", False, 0]
+    idx.add(data[:10])
+    _search(idx, q, 10)
+    assert said() == [False, "lists", False, 0]
+    idx._screening(True)
+    _same(_search(idx, q, 10)[:2], oracle.flat_search(np.concatenate([data, data[:10]]), q, 10,
+                                                      oracle.L2)[:2])
+    assert said() == [True, "screened", False, 1]
+    idx._scan_f16(False)
+    _search(idx, q, 10)
+    assert said() == [False, "lists", False, 0]
+
+    pq = PqIndex(64, Metric.L2, m=16, train_iters=1, train_sample=1000)
+    pq.train(data)
+    pq.add(data)
+    a = pq.search_batch(q, k=10)
+    assert pq._last_timing()["screened"]
+    pq._screening(False)
+    _same(pq.search_batch(q, k=10), a)
+    assert not pq._last_timing()["screened"]
+    pq._screening(True)
+    _same(pq.search_batch(q, k=10), a)
+    assert pq._last_timing()["screened"]
 
 
 def test_results_past_the_mapped_buffer(gpu):

@@ -76,6 +76,7 @@ def _give_up_then_recover(dev, data, q, k, metric, path, f16=False, mask=None,
     lib = dev.lib
     nq = len(q)
     idx = FlatIndex(data.shape[1], Metric.L2 if metric == oracle.L2 else Metric.InnerProduct)
+    idx._screening(False)
     idx.add(data)
     idx._scan_f16(f16)
     dq = dev.put(q)
