@@ -2,7 +2,8 @@
  * A HIP runtime for tests of host code without a GPU, preloaded over the real one: one gfx950
  * device whose memory is the host's, copies done at once, kernels that do nothing (what they
  * would have read back is zero). A launch of a kernel whose name holds the text in
- * PX_STUB_FAIL_LAUNCH fails with hipErrorLaunchFailure.
+ * PX_STUB_FAIL_LAUNCH fails with hipErrorLaunchFailure; launches of kernels whose name holds the
+ * text in PX_STUB_COUNT_LAUNCH are counted in px_stub_launches.
  */
 #define __HIP_PLATFORM_AMD__
 #include <hip/hip_runtime_api.h>
@@ -13,6 +14,7 @@
 static struct { const void* host; const char* name; } kernels[4096];
 static int kernel_count;
 static hipError_t last;
+long px_stub_launches;
 
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
@@ -25,9 +27,28 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int d) {
     return hipSuccess;
 }
 hipError_t hipMemGetInfo(size_t* left, size_t* total) { *left = *total = (size_t)1 << 36; return hipSuccess; }
-hipError_t hipMalloc(void** p, size_t n) { *p = calloc(1, n ? n : 1); return *p ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipFree(void* p) { free(p); return hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) { (void)flags; return hipMalloc(p, n); }
+/* device memory: its size before it, the bytes held in px_stub_live */
+#define HEAD 64
+size_t px_stub_live;
+hipError_t hipMalloc(void** p, size_t n) {
+    char* m = calloc(1, n + HEAD);
+    *p = m ? m + HEAD : 0;
+    if (!m) return last = hipErrorOutOfMemory;
+    *(size_t*)m = n;
+    px_stub_live += n;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+    if (!p) return hipSuccess;
+    px_stub_live -= *(size_t*)((char*)p - HEAD);
+    free((char*)p - HEAD);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
+    (void)flags;
+    *p = calloc(1, n ? n : 1);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned flags) { (void)flags; *d = h; return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned flags) { (void)flags; *s = malloc(1); return hipSuccess; }
@@ -66,7 +87,11 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* m, hipStream_t* s
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t m, hipStream_t s) {
     (void)g, (void)b, (void)args, (void)m, (void)s;
     const char* fail = getenv("PX_STUB_FAIL_LAUNCH");
-    for (int i = 0; fail && *fail && i < kernel_count; ++i)
-        if (kernels[i].host == f && strstr(kernels[i].name, fail)) return last = hipErrorLaunchFailure;
+    const char* count = getenv("PX_STUB_COUNT_LAUNCH");
+    for (int i = 0; i < kernel_count; ++i) {
+        if (kernels[i].host != f) continue;
+        if (count && *count && strstr(kernels[i].name, count)) ++px_stub_launches;
+        if (fail && *fail && strstr(kernels[i].name, fail)) return last = hipErrorLaunchFailure;
+    }
     return hipSuccess;
 }

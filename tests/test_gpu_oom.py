@@ -143,7 +143,7 @@ def test_flat_search_that_fits_without_screening(gpu, budget, copy_kept):
     ids, d = idx.search_batch(q, k=10)
     assert idx._last_timing()["screened"] == copy_kept
     assert np.array_equal(ids, o_ids) and np.array_equal(d, o_d)
-    idx.add(data[:1])  # (room for it: the copy is brought up to date, or made again)
+    idx.add(data[:15_000])  # (room for it: the copy is brought up to date, or made again)
     idx.search_batch(q, k=10)
     assert idx._last_timing()["screened"]
 

@@ -175,6 +175,11 @@ def test_magnitudes(gpu):
         _exact(np.ldexp(data, e), np.ldexp(q, e), 10, oracle.IP)
     idx = _index(np.ldexp(data, 50), oracle.IP)
     assert not _search(idx, q, 10)[2]["screened"]
+    # rows added later may all be smaller than that
+    idx = _index(data, oracle.IP)
+    tiny = np.ldexp(datagen.gaussian(100, 48, 973), -60)
+    idx.add(tiny)
+    _exact(np.concatenate([data, tiny]), q, 10, oracle.IP, idx=idx)
 
 
 def test_queries_whose_residuals_square_to_nothing(gpu):

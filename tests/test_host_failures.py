@@ -1,6 +1,6 @@
-"""What the host code does when a device operation fails, on the CPU: the library on a stand-in
-HIP runtime (tests/c_abi/hip_stub.c) whose kernels do nothing and whose launches fail where a
-test says so."""
+"""What the host code does when a device operation fails, and what it holds, on the CPU: the
+library on a stand-in HIP runtime (tests/c_abi/hip_stub.c) whose kernels do nothing, whose
+launches fail where a test says so and which counts the bytes of device memory."""
 import os
 import subprocess
 import sys
@@ -25,8 +25,18 @@ import os
 import numpy as np
 from proxima_amd import FlatIndex, Metric, PqIndex
 
+import ctypes
+stub = ctypes.CDLL(os.environ["LD_PRELOAD"])
 def fail(name):
     os.environ["PX_STUB_FAIL_LAUNCH"] = name
+def live():
+    return ctypes.c_size_t.in_dll(stub, "px_stub_live").value
+def launches(name, call):
+    n = ctypes.c_long.in_dll(stub, "px_stub_launches")
+    n.value, os.environ["PX_STUB_COUNT_LAUNCH"] = 0, name
+    call()
+    os.environ["PX_STUB_COUNT_LAUNCH"] = ""
+    return n.value
 """
     r = subprocess.run([sys.executable, "-c", head + code], env=dict(os.environ, LD_PRELOAD=stub),
                        capture_output=True, text=True, timeout=120)
@@ -80,4 +90,52 @@ else:
 fail("")
 idx.add(x)
 assert len(idx) == 5000
+""")
+
+
+# The screening copy of an index of codes takes at most 8 GiB, room for more rows counted, and
+# nothing once the rows are past that: 256 bytes a row, 33.5M rows. (The copy is never touched
+# here: the stand-in's kernels do nothing.)
+def test_pq_screening_copy_is_bounded_and_given_back(stub):
+    _run(stub, """
+pq = PqIndex(4, Metric.L2, m=1, train_iters=0, train_sample=256)
+pq.train(np.arange(256 * 4, dtype=np.float32).reshape(256, 4))
+codes = np.zeros((17_000_000, 1), dtype=np.uint8)
+pq.add_codes(codes)
+one = live()
+assert one > 17_000_000 * 256
+pq.add_codes(codes[:10])  # room for 34M codes
+assert 17_000_000 * 256 < live() < (8 << 30) + 34_000_000 * 5 + (1 << 20), live()
+pq.add_codes(codes[:16_600_000])
+assert live() < 68_000_010 + (1 << 20), live()
+""")
+
+
+def test_flat_screening_copy_is_bounded_and_given_back(stub):
+    # 8 dims: 32 bytes a row and 256 of copy
+    _run(stub, """
+idx = FlatIndex(8, Metric.L2)
+x = np.zeros((17_000_000, 8), dtype=np.float32)
+x[0, 0] = 1
+idx.add(x)
+idx.add(x[:16_900_000])  # room for 34M rows: their copy would be 8.7 GB
+assert live() < 34_000_000 * 37 + (1 << 20), live()
+""")
+
+
+def test_pq_copy_that_cannot_be_had_is_not_tried_at_every_search(stub):
+    # device memory for the codes and not for the copy: one try an eighth more rows
+    _run(stub, """
+pq = PqIndex(8, Metric.L2, m=8, train_iters=0, train_sample=256)
+pq.train(np.arange(256 * 8, dtype=np.float32).reshape(256, 8))
+codes = np.zeros((40_000, 8), dtype=np.uint8)
+os.environ["PX_DEVICE_BUDGET"] = str(9_000_000)
+pq.add_codes(codes)
+assert live() < 1_000_000
+del os.environ["PX_DEVICE_BUDGET"]
+q = np.zeros((1, 8), dtype=np.float32)
+assert launches("screen_codes", lambda: [pq.search_batch(q, k=1) for _ in range(5)]) == 0
+assert launches("screen_codes", lambda: pq.add_codes(codes[:10])) == 0
+assert launches("screen_codes", lambda: pq.add_codes(codes[:5000])) == 1
+assert live() > 45_000 * 256
 """)
