@@ -1970,7 +1970,15 @@ __global__ __launch_bounds__(1024) void flat_collect_select_kernel(CollectSelect
     // the kk-th smallest key by a radix select (four 8-bit passes over the order-preserving
     // unsigned form of the total-order key, so the key is exact), then only the candidates
     // at or below it (at least kk, ties included) are compacted and sorted.
-    if (avail > 512 && avail > 2 * a.kk) {
+    // (screened, kk to twice kk of them: where the survivors' sort is the shorter one; 192k x 128,
+    // k = 3,000: a search of one query 304 -> 236 us, of 1,000 3.24 -> 2.90 ms)
+    auto sort_width = [](int n) __attribute__((always_inline)) {
+        int p = 1;
+        while (p < n) p <<= 1;
+        return p;
+    };
+    if (avail > 512 &&
+        (avail > 2 * a.kk || (a.err && sort_width(avail) > sort_width(a.kk + 32)))) {
         __shared__ unsigned rhist[256];
         __shared__ unsigned s_pre, s_need;
         if (t == 0) {

@@ -66,6 +66,15 @@ def test_sizes(gpu, n, dim, nq, k, metric, kind):
     assert info["collect_rounds"] == 1
 
 
+@pytest.mark.parametrize("n,k,nq", [(262_144, 4_096, 20), (192_000, 3_000, 20), (140_000, 2_000, 3),
+                                    (64_000, 1_000, 300), (5_000, 78, 40)])
+def test_most_neighbours(gpu, n, k, nq):
+    # k a 64th of the rows or little less: the sample's threshold still lets no more through than
+    # the select holds, and every query finishes in the first round
+    _, info = _exact(datagen.gaussian(n, 32, 905), datagen.gaussian(nq, 32, 906), k, oracle.L2)
+    assert info["collect_rounds"] == 1, info
+
+
 @pytest.mark.parametrize("dim", [96, 200])
 @pytest.mark.parametrize("metric", [oracle.L2, oracle.IP])
 def test_filtered(gpu, dim, metric):
