@@ -106,6 +106,7 @@ __global__ __launch_bounds__(512) void flat_screen_kernel(ScreenArgs a) {
     __shared__ __attribute__((aligned(16))) char tile[kBufs][kScreenRows * kPitch];
     __shared__ __attribute__((aligned(16))) float tnorm[kNormSlots][kScreenRows];
     __shared__ int committed[8];  // per wave: the last stage it has committed
+    __shared__ int wants[8];      // per wave: whether a row can pass for one of its queries
     // rows each lane has appended for its two queries: in LDS, as registers they spilled
     __shared__ int counts[MIN ? 1 : QB][MIN ? 1 : 512];
 
@@ -134,6 +135,28 @@ __global__ __launch_bounds__(512) void flat_screen_kernel(ScreenArgs a) {
         asm volatile("" : "+v"(v));
         return v;
     };
+
+    // ---- per-query state, [query block]
+    // Padding slots: a NaN, which no D passes. (Not +inf: after a wait that gave up, D may come
+    // of norms never written, +inf among them, and a slot past nq has no region to append to.)
+    const float kNothing = __int_as_float(0x7fc00000);
+    float nct[QB];  // the threshold as a D value: a row passes at or above it
+    auto query_of = [&](int qb) __attribute__((always_inline)) {
+        const int slot = opaque(slot0 + 32 * qb);
+        return a.qlist ? a.qlist[slot < a.nq ? slot : 0] : (slot < a.nq ? slot : 0);
+    };
+    if constexpr (!MIN) {
+        bool want = false;
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+            nct[qb] = kNothing;
+            if (slot0 + 32 * qb < a.nq)
+                nct[qb] = from_total_key(a.thr_key[query_of(qb)]) * (1.0f / kF) * scale;
+            want |= nct[qb] < kInf;
+        }
+        if (__ballot(want) && lane == 0) wants[wave] = 1;
+        else if (lane == 0) wants[wave] = 0;
+    }
 
     // ---- staging: every load unconditional, positions past the split's end clamped to its
     // last row (their sums are not used). Positions fit 32 bits, unsigned: at most 2^31 + 511.
@@ -238,6 +261,19 @@ __global__ __launch_bounds__(512) void flat_screen_kernel(ScreenArgs a) {
     using P1 = std::integral_constant<int, 1>;
     if (tid < 8) committed[tid] = 1;
     __syncthreads();
+    // no query of the workgroup that a row can pass for (the ladder gave them all up): done
+    if constexpr (!MIN) {
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) any |= wants[w];
+        if (!any) {
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb)
+                if (slot0 + 32 * qb < a.nq)
+                    a.cand_count[((int64_t)(slot0 + 32 * qb) * a.splits + split) * 2 + h] = 0;
+            return;
+        }
+    }
 
     // Stage sync: at the end of stage s a wave waits until every wave has committed stage
     // s + 1 before it reads that stage and writes stage s + 2, whose buffer held stage s - 1
@@ -273,28 +309,13 @@ __global__ __launch_bounds__(512) void flat_screen_kernel(ScreenArgs a) {
         return;
     }
 
-    // ---- per-query state, [query block]
     if constexpr (!MIN) {
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) counts[qb][tid] = 0;
     }
-    // Padding slots: a NaN, which no D passes. (Not +inf: after a wait that gave up, D may come
-    // of norms never written, +inf among them, and a slot past nq has no region to append to.)
-    const float kNothing = __int_as_float(0x7fc00000);
-    float nct[QB];  // the threshold as a D value: a row passes at or above it
     float vmax[QB];
-    auto query_of = [&](int qb) __attribute__((always_inline)) {
-        const int slot = opaque(slot0 + 32 * qb);
-        return a.qlist ? a.qlist[slot < a.nq ? slot : 0] : (slot < a.nq ? slot : 0);
-    };
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-        const int q = query_of(qb);
-        vmax[qb] = -kInf;
-        nct[qb] = kNothing;
-        if (!MIN && slot0 + 32 * qb < a.nq)
-            nct[qb] = from_total_key(a.thr_key[q]) * (1.0f / kF) * scale;
-    }
+    for (int qb = 0; qb < QB; ++qb) vmax[qb] = -kInf;
     // The queries lie in fragment order (ScreenArgs::qs), so that a wave's load is 1 KB in one
     // piece: as rows, its 64 lanes touched 32 cache lines for 32 bytes of each, and those
     // loads, not the matrix units, set the pace of several-chunk scans. Buffer loads: a scalar
@@ -638,12 +659,13 @@ __global__ __launch_bounds__(256) void screen_spread_kernel(const unsigned short
                                                             int ds, float* parts) {
     __shared__ float sums[4][64], squares[4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t n = min(rows, (int64_t)256), step = rows / n;
+    const int64_t n = min(rows, (int64_t)256);
     const unsigned short* x = xs + (int64_t)blockIdx.x * 64 + lane;
     float m = 0.f, v2 = 0.f;
 #pragma unroll 8
     for (int64_t i = wave; i < n; i += 4) {
-        const float v = (float)__builtin_bit_cast(_Float16, x[i * step * ds]);
+        // (i rows / n, not i times a whole step: rows of one kind may lie at every third)
+        const float v = (float)__builtin_bit_cast(_Float16, x[i * rows / n * ds]);
         m += v;
         v2 += v * v;
     }

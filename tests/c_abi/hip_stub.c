@@ -61,6 +61,11 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hip
 }
 hipError_t hipGetLastError(void) { const hipError_t e = last; last = hipSuccess; return e; }
 
+hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute a, int v) {
+    (void)f, (void)a, (void)v;
+    return hipSuccess;
+}
+
 void** __hipRegisterFatBinary(const void* data) { (void)data; static void* h; return &h; }
 void __hipUnregisterFatBinary(void** h) { (void)h; }
 void __hipRegisterFunction(void** h, const void* host, char* dev, const char* name, unsigned t,

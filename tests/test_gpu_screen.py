@@ -104,9 +104,9 @@ def test_near_rows_are_the_sampled_ones(gpu):
     # the sample (every 14th row) is near, the rest far: its thresholds admit too few rows
     rng = np.random.default_rng(931)
     n = 60_000
-    data = (rng.standard_normal((n, 24)) + 30).astype(np.float32)
-    data[::n // 4096] = rng.standard_normal((len(data[::n // 4096]), 24))
-    q = rng.standard_normal((80, 24)).astype(np.float32)
+    data = (rng.standard_normal((n, 24)) * 30).astype(np.float32)
+    data[::n // 4096] = rng.standard_normal((len(data[::n // 4096]), 24)) * 2
+    q = (rng.standard_normal((80, 24)) * 2).astype(np.float32)
     _exact(data, q, 900, oracle.L2)
 
 
@@ -125,8 +125,8 @@ def test_ties(gpu):
 @pytest.mark.parametrize("name", ["offset", "query scale", "zero queries", "outlier row"])
 def test_what_screening_leaves_open(gpu, name):
     # the bound spans every row (a large common offset), is infinite (scales 2^45 apart), or is
-    # widened by one row of huge norm: whatever screening finishes or leaves, the results are
-    # the fp32 scans'
+    # widened by one row of huge norm, added later: whatever screening finishes or leaves, the
+    # results are the fp32 scans'
     rng = np.random.default_rng(951)
     data = rng.standard_normal((60_000, 64)).astype(np.float32)
     q = rng.standard_normal((90, 64)).astype(np.float32)
@@ -139,16 +139,22 @@ def test_what_screening_leaves_open(gpu, name):
         q *= np.float32(2.0 ** 45)
     elif name == "zero queries":
         q[::3] = 0
-    else:
-        data[777] = 3e4
     metric = oracle.IP if name == "query scale" else oracle.L2
     idx = _index(data, metric)
+    if name == "outlier row":
+        assert _search(idx, q, 10)[2]["screened"]
+        idx.add(np.full((1, 64), 3e4, dtype=np.float32))
     print(f"case screen left open: {name}", flush=True)
     ids, d, info = _search(idx, q, 10)
     # (rows so far from the origin that fp16 cannot tell them apart are not screened)
     assert info["screened"] == (name != "offset")
     if name == "query scale":
-        assert info["collect_rounds"] >= 2  # and the fp32 collect scan's
+        assert info["collect_rounds"] == 1  # (90 queries: the fp32 lists finish them)
+    # an index on which such a search is no accident is not screened again; one whose rows can be
+    # told apart by queries of their own kind is
+    ids2, d2, info = _search(idx, q, 10)
+    assert info["screened"] == (name in ("query scale", "zero queries"))
+    _same((ids, d), (ids2, d2))
     idx._scan_f16(False)
     ids32, d32, info32 = _search(idx, q, 10)
     assert not info32["screened"]
@@ -159,7 +165,7 @@ def test_rows_added_later(gpu):
     # the copy grows with the rows, is made again when a row passes its scale, and starts when
     # an index gets its 4,096th row or its first row that is not exact in fp16
     a, b = datagen.gaussian(4_000, 72, 961), datagen.gaussian(30_000, 72, 962)
-    big = (datagen.gaussian(2_000, 72, 963) * 4096).astype(np.float32)
+    big = (datagen.gaussian(40_000, 72, 963) * 128).astype(np.float32)
     q = datagen.gaussian(50, 72, 964)
     idx = _index(a, oracle.IP)
     assert not _search(idx, q, 5)[2]["screened"]
@@ -228,14 +234,76 @@ def test_give_up(gpu):
 
 @pytest.mark.parametrize("nq", [3, 300])
 def test_too_many_rows_within_the_bound(gpu, nq):
-    # two tight groups about opposite points: rows spread about the origin, but half of them
-    # within the bound of every query's neighbours; the ladder gives such queries up and the
-    # fp32 path answers (values as in the offset case above)
+    # two thirds of the rows spread widely, a third in one tight group about a far point, all of
+    # it within the bound of the neighbours of queries beside it: the ladder gives such queries
+    # up and the scans without screening answer them; others of the batch are screened (values
+    # near the group as in the offset case above)
     rng = np.random.default_rng(985)
-    sign = np.where(rng.random((30_000, 1)) < 0.5, -1, 1)
-    data = (sign * 128 + np.round(rng.standard_normal((30_000, 64)) * 2) / 2).astype(np.float32)
-    q = (128 + np.round(rng.standard_normal((nq, 64)) * 2) / 2).astype(np.float32)
-    _exact(data, q, 10, oracle.L2)
+    data = np.round(rng.standard_normal((30_000, 64)) * 100).astype(np.float32)
+
+    def tight(n):
+        return 128 + np.round(rng.standard_normal((n, 64)) * 2) / 2
+
+    data[::3] = tight(10_000)  # (a period that a whole step of a row sample would meet)
+    q = tight(nq).astype(np.float32)
+    q[::4] = np.round(rng.standard_normal((len(q[::4]), 64)) * 100)
+    _, info = _exact(data, q, 10, oracle.L2)
+    assert info["collect_rounds"] == (2 if nq == 3 else 1)  # (3: the vector-ALU scan collects)
+
+
+@pytest.mark.parametrize("kind", ["two groups", "fifty groups", "copies"])
+def test_rows_too_close_together_for_screening(gpu, kind):
+    # rows in groups that the bound cannot tell apart, larger than a select is worth: after one
+    # search that screening left open such an index is not screened, until it has other rows too
+    rng = np.random.default_rng(986)
+    centres = {"two groups": 2, "fifty groups": 50, "copies": 16}[kind]
+    c = rng.standard_normal((centres, 64)) * 64
+
+    def near(n):
+        off = rng.standard_normal((n, 64)) / 256 if kind != "copies" else 0
+        return (c[rng.integers(centres, size=n)] + off).astype(np.float32)
+
+    data, q = near(60_000), near(20)
+    idx = _index(data, oracle.L2)
+    first, second = _search(idx, q, 10), _search(idx, q, 10)
+    assert first[2]["screened"] and not second[2]["screened"]
+    _same(first[:2], second[:2])
+    other = (datagen.gaussian(200_000, 64, 987) * 64).astype(np.float32)
+    idx.add(other)
+    assert _search(idx, other[:20], 10)[2]["screened"]
+
+
+def test_rows_exact_in_fp16_too_close_together(gpu):
+    # the same of the fp16 copy of exact rows, whose vector and list routes are screened: copies
+    # of 16 rows
+    rng = np.random.default_rng(989)
+    data = rng.integers(0, 256, size=(16, 128)).astype(np.float32)[rng.integers(16, size=70_000)]
+    q = rng.integers(0, 256, size=(20, 128)).astype(np.float32)
+    idx = _index(data, oracle.L2)
+    o = oracle.flat_search(data, q, 10, oracle.L2)[:2]
+    for screened in (True, False, False):
+        ids, d, info = _search(idx, q, 10)
+        assert info["screened"] == screened
+        _same((ids, d), o)
+    more = rng.integers(0, 256, size=(200_000, 128)).astype(np.float32)
+    idx.add(more)
+    for _ in range(2):
+        ids, d, info = _search(idx, more[:20], 10)
+        assert info["screened"]
+        _same((ids, d), oracle.flat_search(np.concatenate([data, more]), more[:20], 10,
+                                           oracle.L2)[:2])
+
+
+def test_codes_of_few_distinct_rows_are_not_screened(gpu):
+    rng = np.random.default_rng(988)
+    data = rng.standard_normal((100_000, 8)).astype(np.float32)
+    pq = PqIndex(8, Metric.L2, m=1, nbits=8, train_iters=2, train_sample=4000)
+    pq.train(data)
+    pq.add(data)
+    q = rng.standard_normal((20, 8)).astype(np.float32)
+    ids, d, info = _search(pq, q, 10)
+    assert not info["screened"]
+    _same((ids, d), oracle.pq_search(pq.codebooks(), pq.codes(), q, 10, oracle.L2)[:2])
 
 
 # ADC searches: the rows that the codes stand for, screened the same way; a key recomputed as

@@ -98,16 +98,16 @@ assert len(idx) == 5000
 # here: the stand-in's kernels do nothing.)
 def test_pq_screening_copy_is_bounded_and_given_back(stub):
     _run(stub, """
-pq = PqIndex(4, Metric.L2, m=1, train_iters=0, train_sample=256)
+pq = PqIndex(4, Metric.L2, m=4, train_iters=0, train_sample=256)
 pq.train(np.arange(256 * 4, dtype=np.float32).reshape(256, 4))
-codes = np.zeros((17_000_000, 1), dtype=np.uint8)
+codes = np.zeros((17_000_000, 4), dtype=np.uint8)
 pq.add_codes(codes)
 one = live()
 assert one > 17_000_000 * 256
 pq.add_codes(codes[:10])  # room for 34M codes
-assert 17_000_000 * 256 < live() < (8 << 30) + 34_000_000 * 5 + (1 << 20), live()
+assert 17_000_000 * 256 < live() < (8 << 30) + 34_000_000 * 8 + (1 << 20), live()
 pq.add_codes(codes[:16_600_000])
-assert live() < 68_000_010 + (1 << 20), live()
+assert live() < 68_000_010 * 4 + (1 << 20), live()
 """)
 
 
