@@ -3,7 +3,8 @@
  * device whose memory is the host's, copies done at once, kernels that do nothing (what they
  * would have read back is zero). A launch of a kernel whose name holds the text in
  * PX_STUB_FAIL_LAUNCH fails with hipErrorLaunchFailure; launches of kernels whose name holds the
- * text in PX_STUB_COUNT_LAUNCH are counted in px_stub_launches.
+ * text in PX_STUB_COUNT_LAUNCH are counted in px_stub_launches, waits for a stream in
+ * px_stub_waits.
  */
 #define __HIP_PLATFORM_AMD__
 #include <hip/hip_runtime_api.h>
@@ -14,7 +15,7 @@
 static struct { const void* host; const char* name; } kernels[4096];
 static int kernel_count;
 static hipError_t last;
-long px_stub_launches;
+long px_stub_launches, px_stub_waits;
 
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
@@ -52,7 +53,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned flags) { (void)flags; *d = h; return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned flags) { (void)flags; *s = malloc(1); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; ++px_stub_waits; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t st) {
     (void)k, (void)st;

@@ -61,6 +61,27 @@ assert len(idx) == 5008
 """)
 
 
+@pytest.mark.parametrize("kernel", ["abs_max_kernel", "screen_rows_kernel"])
+def test_flat_add_survives_a_failure_beside_it(stub, kernel):
+    # an index with a copy: the rows added go to it in the same pass
+    _run(stub, f"""
+x = np.arange(5000 * 8, dtype=np.float32).reshape(5000, 8)
+idx = FlatIndex(8, Metric.L2)
+idx.add(x)
+idx.add(x[:1])  # (room for 10,000 rows)
+one = live()
+idx.add(x[:1])
+assert live() == one
+fail({kernel!r})
+idx.add(x[:7])
+assert len(idx) == 5009 and live() < one - 10_000 * 256 + (1 << 16)
+fail("")
+idx.add(x[:1000])
+assert len(idx) == 6009 and live() >= one - (1 << 16)
+assert np.array_equal(idx.vectors(), np.concatenate([x, x[:1], x[:1], x[:7], x[:1000]]))
+""")
+
+
 @pytest.mark.parametrize("kernel", ["screen_codes_kernel", "screen_spread_kernel"])
 def test_pq_add_survives_a_failed_screening_copy(stub, kernel):
     _run(stub, f"""
@@ -138,4 +159,24 @@ assert launches("screen_codes", lambda: [pq.search_batch(q, k=1) for _ in range(
 assert launches("screen_codes", lambda: pq.add_codes(codes[:10])) == 0
 assert launches("screen_codes", lambda: pq.add_codes(codes[:5000])) == 1
 assert live() > 45_000 * 256
+""")
+
+
+def test_an_add_of_a_few_rows_waits_no_more_than_without_a_copy(stub):
+    # the waits of the host are what such an add costs
+    _run(stub, """
+def waits(call):
+    n = ctypes.c_long.in_dll(stub, "px_stub_waits")
+    n.value = 0
+    call()
+    return n.value
+x = np.arange(5000 * 8, dtype=np.float32).reshape(5000, 8)
+n = []
+for screening in (False, True):
+    idx = FlatIndex(8, Metric.L2)
+    idx._screening(screening)
+    idx.add(x)
+    idx.add(x[:1])
+    n.append(waits(lambda: idx.add(x[:1])))
+assert n[0] == n[1] == 1, n
 """)
