@@ -354,6 +354,36 @@ def test_device_query_nonfinite_leaves_outputs(gpu, nq, k, masked, path):
             lib.px_dev_free(p)
 
 
+def test_device_query_nonfinite_in_a_later_batch(gpu):
+    # more queries than one screening pass takes (16,384): an infinite value in the last leaves the
+    # outputs of all of them unwritten
+    lib = _lib.load()
+    nq, k = 16_400, 2
+    data = datagen.gaussian(5_000, 8, 47)
+    q = datagen.gaussian(nq, 8, 48)
+    q[-1, 3] = np.inf
+    idx = FlatIndex(8, Metric.L2)
+    idx.add(data)
+    ids = np.full((nq, k), 1234567, dtype=np.int64)
+    d = np.full((nq, k), 7.5, dtype=np.float32)
+    ptrs = []
+    try:
+        for a in (q, ids, d):
+            p = ctypes.c_void_p()
+            assert lib.px_dev_alloc(ctypes.byref(p), a.nbytes) == 0
+            ptrs.append(p)
+            assert lib.px_dev_upload(p, a.ctypes.data, a.nbytes) == 0
+        print("case nonfinite device query in the second batch", flush=True)
+        rc = lib.px_flat_search_device(idx._h, ptrs[0], nq, k, None, ptrs[1], ptrs[2])
+        assert rc == _lib.PX_ERR_NONFINITE, (rc, _lib.last_error())
+        assert lib.px_dev_download(ids.ctypes.data, ptrs[1], ids.nbytes) == 0
+        assert lib.px_dev_download(d.ctypes.data, ptrs[2], d.nbytes) == 0
+        assert (ids == 1234567).all() and (d == 7.5).all()
+    finally:
+        for p in ptrs:
+            lib.px_dev_free(p)
+
+
 @pytest.mark.parametrize("k", [24, 25, 48, 49, 112, 113, 120])
 def test_list_capacity_boundaries(gpu, k):
     # k' = k + 8 crosses the list classes (32 int ids | 56 and 120 with 16-bit offsets | 128)
