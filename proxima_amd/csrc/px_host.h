@@ -4,7 +4,6 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -55,14 +54,14 @@ void parallel_for(int64_t n, F&& body) {
     const int nt = (int)std::min<int64_t>(host_threads(), std::max<int64_t>(n, 1));
     const int64_t per = (n + nt - 1) / nt;
     std::vector<std::thread> th;
-    th.reserve(nt);
     int64_t lo = per;
     try {
+        th.reserve(nt);
         for (; lo < n; lo += per) {
             const int64_t hi = std::min(n, lo + per);
             th.emplace_back([&body, lo, hi] { body(lo, hi); });
         }
-    } catch (const std::system_error&) {
+    } catch (...) {  // (no thread, or no memory for one)
     }
     body(0, std::min(per, n));
     if (lo < n) body(lo, n);

@@ -11,7 +11,29 @@ CSRC = os.path.join(os.path.dirname(HERE), "proxima_amd", "csrc")
 
 SHIM = r"""
 #include "px_host.h"
+#include <atomic>
+#include <cstdlib>
+#include <new>
+// allocations fail from the nth on, where n is set
+static std::atomic<int> left{-1};
+void* operator new(std::size_t n) {
+    if (left.load() >= 0 && left.fetch_sub(1) <= 0) throw std::bad_alloc();
+    return std::malloc(n);
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+namespace px { int host_threads() { return 4; } }
 extern "C" {
+// the sum of [0, n) by parallel_for; at most `allocations` of its allocations succeed (-1: all)
+int64_t parallel_sum(int64_t n, int allocations) {
+    std::atomic<int64_t> sum{0};
+    left = allocations;
+    px::parallel_for(n, [&](int64_t lo, int64_t hi) {
+        for (int64_t i = lo; i < hi; ++i) sum += i;
+    });
+    left = -1;
+    return sum.load();
+}
 int64_t ref_roundings(int64_t n) { return px::ref_roundings(n); }
 int64_t screen_batch(int64_t ds, int64_t most) { return px::screen_batch(ds, most); }
 int screen_batch_fits(int64_t nq, int64_t ds) { return px::screen_batch_fits(nq, ds); }
@@ -24,11 +46,13 @@ def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("screen_host")
     src, out = d / "shim.cpp", d / "shim.so"
     src.write_text(SHIM)
-    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-I", CSRC, "-o", str(out),
-                    str(src), "-lpthread"], check=True, timeout=120)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wl,-Bsymbolic", "-I", CSRC,
+                    "-o", str(out), str(src), "-lpthread"], check=True, timeout=120)
     lib = ctypes.CDLL(str(out))
     lib.ref_roundings.restype = ctypes.c_int64
     lib.ref_roundings.argtypes = [ctypes.c_int64]
+    lib.parallel_sum.restype = ctypes.c_int64
+    lib.parallel_sum.argtypes = [ctypes.c_int64, ctypes.c_int]
     lib.screen_batch.restype = ctypes.c_int64
     for f in (lib.screen_batch, lib.screen_batch_fits):
         f.argtypes = [ctypes.c_int64, ctypes.c_int64]
@@ -83,3 +107,11 @@ def test_screen_batch_is_what_the_scan_takes(lib):
         assert lib.screen_batch(ds, 1000) == min(b, 1000)
     assert 0 in seen and 16_384 in seen and len(seen) > 4
     assert not lib.screen_batch_fits(16_384, 63_616)  # one launch of the whole batch is refused
+
+
+def test_parallel_for_without_memory_for_threads(lib):
+    # a host pass over a caller's data is at the C ABI's entries: where threads cannot be had, for
+    # whatever reason, the calling thread does the rest
+    for allocations in (-1, 0, 1, 2, 3):
+        for n in (0, 1, 3, 4, 1001):
+            assert lib.parallel_sum(n, allocations) == n * (n - 1) // 2, (n, allocations)
