@@ -23,6 +23,13 @@ def test_host_code_under_sanitizers():
     build = subprocess.run(["make", "-s", "-C", os.path.join(HERE, "c_abi"), "sanitize"],
                            capture_output=True, text=True, timeout=900)
     assert build.returncode == 0, build.stderr[-4000:]
+    # the library is whole: a symbol of its own left to lazy binding would only be missed by the
+    # first call that needs it (the sanitizers' come from the executable)
+    nm = subprocess.run(["nm", "-D", "-u", "--demangle",
+                         os.path.join(ROOT, "_build", "asan", "libproxima_px_asan.so")],
+                        capture_output=True, text=True, timeout=60)
+    assert nm.returncode == 0, nm.stderr
+    assert "px::" not in nm.stdout, nm.stdout
     env = dict(os.environ,
                ASAN_OPTIONS="detect_leaks=1",
                LSAN_OPTIONS="suppressions=" + os.path.join(HERE, "c_abi", "lsan.supp"),
