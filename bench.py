@@ -591,23 +591,27 @@ def pq_measure(args, dev, pq, queries, mask, n, m, nq, k):
 
     # value and ms_per_step from searches as a caller makes them, then the same searches with
     # the library's HIP events on for the kernel and pipeline times
-    pq._timing(False)
-    for _ in range(args.warmup):
+    def timed():
+        pq._timing(False)
+        for _ in range(args.warmup):
+            step()
+        t0 = time.perf_counter()
+        for _ in range(args.steps):
+            step()
+        elapsed = time.perf_counter() - t0
+        pq._timing(True)
         step()
-    t0 = time.perf_counter()
-    for _ in range(args.steps):
-        step()
-    elapsed = time.perf_counter() - t0
-    pq._timing(True)
-    step()
-    scan_ms, total_ms = [], []
-    for _ in range(args.steps):
-        step()
-        read_timing(*timing_args)
-        scan_ms.append(ev_scan.value)
-        total_ms.append(ev_total.value)
+        scan, total = [], []
+        for _ in range(args.steps):
+            step()
+            read_timing(*timing_args)
+            scan.append(ev_scan.value)
+            total.append(ev_total.value)
+        pq._timing(False)
+        return elapsed, scan, total
+
+    elapsed, scan_ms, total_ms = timed()
     screened = pq._last_timing()["screened"]
-    pq._timing(False)
     ids = dev.get(di, np.empty((nq, k), dtype=np.int64))
     dists = dev.get(dd, np.empty((nq, k), dtype=np.float32))
     if mask is not None:
@@ -654,6 +658,23 @@ def pq_measure(args, dev, pq, queries, mask, n, m, nq, k):
                               "kernel": "flat_screen_kernel",
                               "kernel_ms": float(np.mean(scan_ms)),
                               "algorithmic_flop_per_launch": flops}
+        # and on the lookup tables, which serve what is not screened
+        pq._screening(False)
+        el_lut, scan_lut, total_lut = timed()
+        lut_ids = dev.get(di, np.empty((nq, k), dtype=np.int64))
+        lut_d = dev.get(dd, np.empty((nq, k), dtype=np.float32))
+        pq._screening(True)
+        result["lut_scan"] = {"value": nq * args.steps / el_lut, "unit": "queries/s",
+                              "ms_per_step": el_lut / args.steps * 1e3, "kernel": "pq_scan_kernel",
+                              "kernel_ms": float(np.mean(scan_lut)),
+                              "pipeline_ms": float(np.mean(total_lut)),
+                              "same_results_as_screened": bool(
+                                  np.array_equal(lut_ids, ids) and
+                                  np.array_equal(lut_d.view(np.uint32), dists.view(np.uint32)))}
+        pq_lds_roofline(result["lut_scan"], mask, nq, n_eff, m, scan_lut, headline_shape)
+        log(f"[bench] PQ LUT scan: {el_lut / args.steps * 1e3:.3f} ms a batch, scan "
+            f"{np.mean(scan_lut):.3f} ms, same results "
+            f"{result['lut_scan']['same_results_as_screened']}")
     else:
         pq_lds_roofline(result, mask, nq, n_eff, m, scan_ms, headline_shape)
     if args.latency > 0 and mask is None:
