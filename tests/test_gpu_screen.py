@@ -190,6 +190,11 @@ def test_magnitudes(gpu):
         _exact(np.ldexp(data, e), np.ldexp(q, e), 10, oracle.IP)
     idx = _index(np.ldexp(data, 50), oracle.IP)
     assert not _search(idx, q, 10)[2]["screened"]
+    # ... added later too, where the copy's scale could still carry them
+    idx = _index(np.ldexp(data, 37), oracle.IP)
+    assert _search(idx, q, 10)[2]["screened"]
+    idx.add(np.ldexp(data[:100], 42))
+    assert not _search(idx, q, 10)[2]["screened"]
     # rows added later may all be smaller than that
     idx = _index(data, oracle.IP)
     tiny = np.ldexp(datagen.gaussian(100, 48, 973), -60)
