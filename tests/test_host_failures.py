@@ -26,7 +26,7 @@ import numpy as np
 from proxima_amd import FlatIndex, Metric, PqIndex
 
 import ctypes
-stub = ctypes.CDLL(os.environ["LD_PRELOAD"])
+stub = ctypes.CDLL(os.environ["LD_PRELOAD"].split(":")[0])
 def fail(name):
     os.environ["PX_STUB_FAIL_LAUNCH"] = name
 def live():
@@ -38,8 +38,10 @@ def launches(name, call):
     os.environ["PX_STUB_COUNT_LAUNCH"] = ""
     return n.value
 """
-    r = subprocess.run([sys.executable, "-c", head + code], env=dict(os.environ, LD_PRELOAD=stub),
-                       capture_output=True, text=True, timeout=120)
+    preload = ":".join([stub, *filter(None, [os.environ.get("LD_PRELOAD")])])
+    r = subprocess.run([sys.executable, "-c", head + code],
+                       env=dict(os.environ, LD_PRELOAD=preload), capture_output=True, text=True,
+                       timeout=120)
     assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-4000:])
 
 
